@@ -14,6 +14,7 @@
 #include <algorithm>
 
 #include "gemm.hpp"
+#include "gemm_dev.hpp"
 
 namespace {
 
@@ -23,37 +24,10 @@ constexpr int kBM = 128, kBN = 128, kBK = 64, kGemmThreads = 256;
 static_assert(kBM == kGemmBf16RowTile && kBK == kGemmBf16KStep, "causal_pv_columns follows this tiling");
 constexpr int kLdsRow = kBK + 8;  // bf16 per LDS row (144 bytes)
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 __device__ inline const uint16_t* row_ptr(const uint16_t* base, uint64_t ld, uint64_t ld_hi, uint32_t group,
                                           uint32_t m) {
   if (group) return base + static_cast<uint64_t>(m / group) * ld_hi + static_cast<uint64_t>(m % group) * ld;
   return base + static_cast<uint64_t>(m) * ld;
-}
-
-// Two f32 -> packed bf16 pair, round to nearest even (v_cvt_pk_bf16_f32).
-__device__ inline uint32_t pack_bf16(float lo, float hi) {
-  const bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-  return __builtin_bit_cast(uint32_t, v);
-}
-
-// One Q4 word (8 nibbles, nibble j = column j) -> 8 bf16(s*q + b) in column
-// order. s*q is exact in f32 (8-bit by 4-bit significands), so the fma rounds
-// once, exactly like the reference's separate multiply and add.
-__device__ inline uint4 dequant_word(uint32_t w, float s, float b) {
-  uint32_t lo = w & 0x0F0F0F0Fu;         // columns 0, 2, 4, 6 in bytes 0..3
-  uint32_t hi = (w >> 4) & 0x0F0F0F0Fu;  // columns 1, 3, 5, 7
-  // Hide the masks from the optimiser so each byte converts with one
-  // v_cvt_f32_ubyteN instead of a bit-field extract plus a convert.
-  asm("" : "+v"(lo), "+v"(hi));
-  uint4 r;
-  r.x = pack_bf16(fmaf(s, static_cast<float>(lo & 0xffu), b), fmaf(s, static_cast<float>(hi & 0xffu), b));
-  r.y = pack_bf16(fmaf(s, static_cast<float>((lo >> 8) & 0xffu), b), fmaf(s, static_cast<float>((hi >> 8) & 0xffu), b));
-  r.z = pack_bf16(fmaf(s, static_cast<float>((lo >> 16) & 0xffu), b), fmaf(s, static_cast<float>((hi >> 16) & 0xffu), b));
-  r.w = pack_bf16(fmaf(s, static_cast<float>(lo >> 24), b), fmaf(s, static_cast<float>(hi >> 24), b));
-  return r;
 }
 
 // 8 bf16 at columns [k, k+8) of a row; columns >= K read as zero.
@@ -275,12 +249,6 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmArgs g) {
 // (lanes = 16 rows x 4 chunks) both run at the full LDS rate on gfx950.
 constexpr int kQ4Threads = 512, kQ4Stages = 3;
 constexpr uint32_t kQ4BBytes = 128 * 128;
-constexpr uint32_t kBufferWord3 = 0x00020000;  // raw buffer descriptor, 32-bit data format
-
-__device__ inline __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, kBufferWord3);
-}
-
 // DENSE: every segment has its prepared bf16 copy (GemmQ4::dense, the values
 // dequant_word produces), staged as is: the same LDS tile, hence the same
 // results bit for bit, without the per-tile dequantisation.
@@ -543,22 +511,6 @@ __global__ __launch_bounds__(kQ4Threads) void gemm_q4_kernel(const GemmArgs g) {
 // outside the buffer range and read as zero (their row offset is in the
 // range-checked per-lane offset).
 constexpr int kDmaThreads = 512, kDmaBK = 32;
-constexpr uint32_t kLdsBytes = 160 * 1024;
-
-// One direct-to-LDS load: 16 bytes per lane at LDS address m0 + 16 * lane.
-// m0 is written only here; nothing else in the kernel reads it (no indirect
-// register indexing or GWS / ordered-count operations).
-__device__ inline void lds_load16(__amdgpu_buffer_rsrc_t r, uint32_t lds_addr, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :
-               : "s"(lds_addr), "v"(voff), "s"(r), "s"(soff)
-               : "memory", "m0");
-}
-// s_waitcnt with vmcnt <= n and the other counters left alone (gfx9 encoding:
-// vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
-#define PRG_WAIT_VMCNT(n) \
-  __builtin_amdgcn_s_waitcnt(((n) & 15) | (7 << 4) | (15 << 8) | ((((n) >> 4) & 3) << 14))
-
 template <int EPI, int BM>
 __global__ __launch_bounds__(kDmaThreads) void gemm_dma_kernel(const GemmArgs g) {
   static_assert(BM == 256 || BM == 320, "row tile");
@@ -777,6 +729,10 @@ int launch_q4_t(hipStream_t s, const GemmArgs& g, const char* name) {
     const uint32_t blocks = ((g.M + bm - 1) / bm) * tiles_n;
     return static_cast<uint64_t>((blocks + cus - 1) / cus) * bm;
   };
+  const uint64_t cold = std::min(cost(192), cost(256));
+  // Few rows: where blocks of 16 to 128 weight rows take fewer units than the
+  // best of the row-tiled kernels (a PEREGRINE_GEMM_DMA override keeps those).
+  const uint64_t small = dma_override() < 0 ? gemm_small_cost(g, EPI, cus) : ~0ull;
   if constexpr (EPI == kGemmSiluPair || EPI == kGemmStore) {
     bool dense = true;
     for (uint32_t i = 0; i < g.nq; ++i) dense = dense && g.q[i].dense != nullptr;
@@ -793,13 +749,13 @@ int launch_q4_t(hipStream_t s, const GemmArgs& g, const char* name) {
         return static_cast<uint64_t>((blocks + cus - 1) / cus) * round;
       };
       const uint64_t c256 = cost_dma(256, kDmaRoundCost256), c320 = cost_dma(320, kDmaRoundCost320);
-      const uint64_t cold = std::min(cost(192), cost(256));
       int pick = dma_override();
-      if (pick < 0) pick = std::min(c256, c320) < cold ? (c320 < c256 ? 320 : 256) : 0;
+      if (pick < 0) pick = std::min(c256, c320) < std::min(cold, small) ? (c320 < c256 ? 320 : 256) : 0;
       if (pick == 320) return launch_dma<EPI, 320>(s, g, tiles_nd, name);
       if (pick == 256) return launch_dma<EPI, 256>(s, g, tiles_nd, name);
     }
   }
+  if (small < cold) return launch_gemm_small(s, g, EPI, cus, name);
   if (cost(192) < cost(256)) return launch_q4_bm<EPI, 192>(s, g, tiles_n, name);
   return launch_q4_bm<EPI, 256>(s, g, tiles_n, name);
 }
