@@ -5,10 +5,7 @@
 //       shaders/linear.metal:780-988 (host Q4Linear.encodePrefillQmm*, linear_q4.zig:197-233)
 //   the prepared-dense route (q4_dequantize_bf16 + MLX bf16 NT GEMM), same numbers
 //       src/model/mlx_nt.zig:139-162
-//   attention score / value GEMMs of the materialised prefill
-//       src/model/block_attn.zig:75-109, 500-631
-//   silu_mul_pair_inplace_bf16 / sigmoid_mul_pair_inplace_bf16 as epilogues
-//       shaders/elementwise.metal:64-99
+//   silu_mul_pair_inplace_bf16 as an epilogue, shaders/elementwise.metal:64-73
 #include <stdlib.h>
 
 #include <algorithm>
@@ -20,217 +17,7 @@ namespace {
 
 using namespace prg;
 
-constexpr int kBM = 128, kBN = 128, kBK = 64, kGemmThreads = 256;
-static_assert(kBM == kGemmBf16RowTile && kBK == kGemmBf16KStep, "causal_pv_columns follows this tiling");
-constexpr int kLdsRow = kBK + 8;  // bf16 per LDS row (144 bytes)
-
-__device__ inline const uint16_t* row_ptr(const uint16_t* base, uint64_t ld, uint64_t ld_hi, uint32_t group,
-                                          uint32_t m) {
-  if (group) return base + static_cast<uint64_t>(m / group) * ld_hi + static_cast<uint64_t>(m % group) * ld;
-  return base + static_cast<uint64_t>(m) * ld;
-}
-
-// 8 bf16 at columns [k, k+8) of a row; columns >= K read as zero.
-__device__ inline uint4 load8(const uint16_t* row, uint32_t k, uint32_t K) {
-  if (!row) return make_uint4(0, 0, 0, 0);
-  if (k + 8 <= K) return *reinterpret_cast<const uint4*>(row + k);
-  uint32_t v[4] = {0, 0, 0, 0};
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    if (k + e < K) v[e >> 1] |= static_cast<uint32_t>(row[k + e]) << (16 * (e & 1));
-  return make_uint4(v[0], v[1], v[2], v[3]);
-}
-
-template <bool Q4, int EPI>
-__global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmArgs g) {
-  // two LDS stages: step k's tiles are read by the matrix cores while step
-  // k+1's are written
-  __shared__ __attribute__((aligned(16))) uint16_t sA[2][kBM * kLdsRow];
-  __shared__ __attribute__((aligned(16))) uint16_t sB[2][kBN * kLdsRow];
-  constexpr bool kPair = (EPI == kGemmSiluPair);
-  constexpr uint32_t kTileN = kPair ? kBN / 2 : kBN;  // output columns per block
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const uint32_t tiles_m = (g.M + kBM - 1) / kBM;
-  const uint32_t tn = blockIdx.x / tiles_m;
-  uint32_t seg = 0;  // Q4 weight segment of this output tile
-  if constexpr (Q4 && !kPair) {
-#pragma unroll
-    for (int i = 1; i < kGemmMaxSegs; ++i)
-      if (i < static_cast<int>(g.nq) && tn >= g.q[i].tile0) seg = i;
-  }
-  const uint32_t m0 = (blockIdx.x % tiles_m) * kBM;
-  const uint32_t n0 = (tn - (Q4 ? g.q[seg].tile0 : 0)) * kTileN;
-  const uint32_t N = Q4 ? g.q[seg].n : g.N;
-  const uint64_t z = blockIdx.z;
-  const uint32_t K = g.K;
-  // Causal attention: the last column any row of this tile sees (rows of one
-  // tile may span two q heads; then the tile holds token T - 1).
-  uint32_t k_end = K;
-  if (!Q4 && g.causal_T != 0) {
-    const uint32_t last = g.causal_prefix + min(g.causal_T - 1, m0 % g.causal_T + (kBM - 1));
-    if (EPI == kGemmStore && n0 > last) return;  // scores: every column masked
-    if (EPI == kGemmSigmoidGate) k_end = causal_pv_columns(m0, g.causal_T, g.causal_prefix, K);  // P.V: zeros past it
-  }
-
-  // Global -> register staging. A (and bf16 B): 16-byte chunk i of this
-  // thread is row (tid/8 + 32 i), columns k0 + 8*(tid%8) .. +8.
-  const int ld_row = tid >> 3, ld_c8 = (tid & 7) * 8;
-  const uint16_t* a_row[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t m = m0 + ld_row + 32 * i;
-    a_row[i] = m < g.M ? row_ptr(g.a + z * g.a_z, g.lda, g.lda_hi, g.a_group, m) : nullptr;
-  }
-  uint4 ra[4];
-  // Q4 B: thread owns tile row tid/2 and half tid%2 of each 64-column group.
-  const int q_row = tid >> 1, q_half = tid & 1;
-  const uint32_t* q_w = nullptr;
-  const uint16_t *q_s = nullptr, *q_b = nullptr;
-  const uint16_t* b_row[4];
-  uint4 rb[4];
-  uint4 rw = make_uint4(0, 0, 0, 0);
-  uint16_t rs = 0, rbias = 0;
-  if constexpr (Q4) {
-    const GemmQ4& Q = g.q[kPair ? (q_row >> 6) : seg];
-    const uint32_t n = n0 + (kPair ? (q_row & 63) : q_row);
-    if (n < N) {
-      q_w = Q.w + static_cast<uint64_t>(n) * (K / 8) + q_half * 4;
-      q_s = Q.s + static_cast<uint64_t>(n) * (K / 64);
-      q_b = Q.b + static_cast<uint64_t>(n) * (K / 64);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t n = n0 + ld_row + 32 * i;
-      b_row[i] = n < N ? g.b + z * g.b_z + static_cast<uint64_t>(n) * g.ldb : nullptr;
-    }
-  }
-
-  auto load = [&](uint32_t k0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ra[i] = load8(a_row[i], k0 + ld_c8, K);
-    if constexpr (Q4) {
-      if (q_w) {
-        rw = *reinterpret_cast<const uint4*>(q_w + k0 / 8);
-        rs = q_s[k0 / 64];
-        rbias = q_b[k0 / 64];
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) rb[i] = load8(b_row[i], k0 + ld_c8, K);
-    }
-  };
-
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // Fragment rows: 16x32 A block i of this wave, 16x32 B block j.
-  const int frow = lane & 15, fk = (lane >> 4) * 8;
-  int brow[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) brow[j] = kPair ? ((j < 2) ? wn * 32 + 16 * j : 64 + wn * 32 + 16 * (j - 2)) : wn * 64 + 16 * j;
-
-  // Registers -> LDS stage st (A as loaded, Q4 B dequantised once here).
-  auto store_stage = [&](int st) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(&sA[st][(ld_row + 32 * i) * kLdsRow + ld_c8]) = ra[i];
-    if constexpr (Q4) {
-      const float s = bf2f(rs), b = bf2f(rbias);
-      uint4* dst = reinterpret_cast<uint4*>(&sB[st][q_row * kLdsRow + q_half * 32]);
-      dst[0] = dequant_word(rw.x, s, b);
-      dst[1] = dequant_word(rw.y, s, b);
-      dst[2] = dequant_word(rw.z, s, b);
-      dst[3] = dequant_word(rw.w, s, b);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(&sB[st][(ld_row + 32 * i) * kLdsRow + ld_c8]) = rb[i];
-    }
-  };
-
-  // One barrier per K step: step k+1 is stored into the other stage and step
-  // k+2's global loads are issued before the matrix cores run on stage k; the
-  // barrier then both publishes stage k+1 and retires the reads of stage k.
-  load(0);
-  store_stage(0);
-  if (kBK < k_end) load(kBK);
-  __syncthreads();
-  int st = 0;
-  for (uint32_t k0 = 0; k0 < k_end; k0 += kBK, st ^= 1) {
-    if (k0 + kBK < k_end) {
-      store_stage(st ^ 1);
-      if (k0 + 2 * kBK < k_end) load(k0 + 2 * kBK);
-    }
-    const uint16_t* A = sA[st];
-    const uint16_t* B = sB[st];
-#pragma unroll
-    for (int kk = 0; kk < kBK; kk += 32) {
-      bf16x8 af[4], bfr[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        af[i] = *reinterpret_cast<const bf16x8*>(&A[(wm * 64 + 16 * i + frow) * kLdsRow + kk + fk]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bfr[j] = *reinterpret_cast<const bf16x8*>(&B[(brow[j] + frow) * kLdsRow + kk + fk]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-
-  // Epilogue: lane holds rows 4*(lane/16) + r, column lane%16 of each block.
-  const int crow = 4 * (lane >> 4), ccol = lane & 15;
-  // Q4: segment output [M, n] row-major; bf16: two-level rows, z offset.
-  uint16_t* C = Q4 ? g.q[seg].c : g.c + z * g.c_z;
-  const uint16_t* R = g.res ? (Q4 ? g.res : g.res + z * g.c_z) : nullptr;
-  const uint64_t ldc = Q4 ? N : g.ldc, ldc_hi = Q4 ? 0 : g.ldc_hi;
-  const uint32_t c_group = Q4 ? 0 : g.c_group;
-  if constexpr (kPair) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t m = m0 + wm * 64 + 16 * i + crow + r;
-        if (m >= g.M) continue;
-        uint16_t* out = const_cast<uint16_t*>(row_ptr(C, ldc, ldc_hi, c_group, m));
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const uint32_t n = n0 + wn * 32 + 16 * j + ccol;
-          if (n >= N) continue;
-          const float gate = round_bf(acc[i][j][r]), up = round_bf(acc[i][j + 2][r]);
-          out[n] = f2bf(silu(gate) * up);
-        }
-      }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t m = m0 + wm * 64 + 16 * i + crow + r;
-        if (m >= g.M) continue;
-        uint16_t* out = const_cast<uint16_t*>(row_ptr(C, ldc, ldc_hi, c_group, m));
-        const uint16_t* rin = R ? row_ptr(R, ldc, ldc_hi, c_group, m) : nullptr;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t n = n0 + wn * 64 + 16 * j + ccol;
-          if (n >= N) continue;
-          const float v = acc[i][j][r];
-          if constexpr (EPI == kGemmStore) {
-            out[n] = f2bf(v);
-          } else if constexpr (EPI == kGemmResidual) {
-            out[n] = f2bf(round_bf(v) + bf2f(rin[n]));
-          } else {
-            out[n] = f2bf(round_bf(v) * sigmoid(bf2f(rin[n])));
-          }
-        }
-      }
-  }
-}
+constexpr int kBN = 128, kBK = 64;  // weight rows per tile and k per step of gemm_q4_kernel
 
 // ---------------------------------------------------------------------------
 // Q4 weights: BM-row x 128-weight-row tiles (BM = 256 or 192), 8 waves (4 along
@@ -760,27 +547,14 @@ int launch_q4_t(hipStream_t s, const GemmArgs& g, const char* name) {
   return launch_q4_bm<EPI, 256>(s, g, tiles_n, name);
 }
 
-template <bool Q4, int EPI>
-int launch_t(hipStream_t s, const GemmArgs& g, uint32_t batch, const char* name) {
-  constexpr uint32_t kTileN = (EPI == kGemmSiluPair) ? kBN / 2 : kBN;
-  uint32_t tiles_n = (g.N + kTileN - 1) / kTileN;
-  if (Q4) tiles_n = (EPI == kGemmSiluPair) ? (g.q[0].n + kTileN - 1) / kTileN : g.q[g.nq - 1].tile0 +
-                    (g.q[g.nq - 1].n + kTileN - 1) / kTileN;
-  const uint32_t tiles = ((g.M + kBM - 1) / kBM) * tiles_n;
-  hipLaunchKernelGGL((gemm_kernel<Q4, EPI>), dim3(tiles, 1, batch), dim3(kGemmThreads), 0, s, g);
-  PRG_CHECK_LAUNCH(name);
-  return PRG_OK;
-}
-
 int check_common(const GemmArgs& g, int epi, const char* name) {
   PRG_CHECK_ARG(g.a, "%s: null A", name);
   PRG_CHECK_ARG(g.M > 0 && g.N > 0 && g.K > 0, "%s: empty problem M=%u N=%u K=%u", name, g.M, g.N, g.K);
-  PRG_CHECK_ARG(g.lda % 8 == 0 && g.lda_hi % 8 == 0 && g.a_z % 8 == 0,
-                "%s: A row strides must be multiples of 8 elements", name);
+  PRG_CHECK_ARG(g.lda % 8 == 0, "%s: A row strides must be multiples of 8 elements", name);
   PRG_CHECK_ARG(reinterpret_cast<uintptr_t>(g.a) % 16 == 0, "%s: A must be 16-byte aligned", name);
-  PRG_CHECK_ARG(epi >= kGemmStore && epi <= kGemmSigmoidGate, "%s: bad epilogue %d", name, epi);
-  PRG_CHECK_ARG((epi != kGemmResidual && epi != kGemmSigmoidGate) || g.res, "%s: epilogue needs res", name);
-  PRG_CHECK_ARG(static_cast<uint64_t>((g.M + kBM - 1) / kBM) * ((g.N + kBN - 1) / kBN) * 2 < (1ull << 31),
+  PRG_CHECK_ARG(epi >= kGemmStore && epi <= kGemmSiluPair, "%s: bad epilogue %d", name, epi);
+  PRG_CHECK_ARG(epi != kGemmResidual || g.res, "%s: epilogue needs res", name);
+  PRG_CHECK_ARG(static_cast<uint64_t>((g.M + 127) / 128) * ((g.N + kBN - 1) / kBN) * 2 < (1ull << 31),
                 "%s: grid too large", name);
   return PRG_OK;
 }
@@ -824,7 +598,6 @@ int launch_gemm_q4(hipStream_t s, GemmArgs g, int epi, const char* name) {
   PRG_CHECK_ARG(g.nq >= 1 && g.nq <= kGemmMaxSegs, "%s: %u weight segments", name, g.nq);
   PRG_CHECK_ARG(epi != kGemmSiluPair || g.nq == 2, "%s: the SiLU pair takes exactly two weights", name);
   PRG_CHECK_ARG(epi != kGemmResidual || g.nq == 1, "%s: the residual epilogue takes one weight", name);
-  PRG_CHECK_ARG(epi != kGemmSigmoidGate, "%s: the sigmoid gate epilogue takes bf16 B", name);
   uint32_t tile = 0;
   g.N = 0;
   for (uint32_t i = 0; i < g.nq; ++i) {
@@ -849,26 +622,10 @@ int launch_gemm_q4(hipStream_t s, GemmArgs g, int epi, const char* name) {
                                     reinterpret_cast<uintptr_t>(g.q[i].dense) % 16 == 0),
                   "%s: prepared bf16 copy of segment %u too large or misaligned", name, i);
   }
-  PRG_CHECK_ARG(g.a_group == 0 && g.a_z == 0, "%s: Q4 GEMM takes plain [M, K] activations", name);
   switch (epi) {
     case kGemmStore: return launch_q4_t<kGemmStore>(s, g, name);
     case kGemmResidual: return launch_q4_t<kGemmResidual>(s, g, name);
     default: return launch_q4_t<kGemmSiluPair>(s, g, name);
-  }
-}
-
-int launch_gemm_bf16(hipStream_t s, const GemmArgs& g, int epi, uint32_t batch, const char* name) {
-  if (int rc = check_common(g, epi, name)) return rc;
-  PRG_CHECK_ARG(g.c, "%s: null C", name);
-  PRG_CHECK_ARG(g.b, "%s: null B", name);
-  PRG_CHECK_ARG(epi != kGemmSiluPair, "%s: the SiLU pair epilogue takes Q4 weights", name);
-  PRG_CHECK_ARG(g.ldb % 8 == 0 && g.b_z % 8 == 0 && reinterpret_cast<uintptr_t>(g.b) % 16 == 0,
-                "%s: B rows must be 16-byte aligned", name);
-  PRG_CHECK_ARG(batch >= 1 && batch <= 65535, "%s: batch %u", name, batch);
-  switch (epi) {
-    case kGemmStore: return launch_t<false, kGemmStore>(s, g, batch, name);
-    case kGemmResidual: return launch_t<false, kGemmResidual>(s, g, batch, name);
-    default: return launch_t<false, kGemmSigmoidGate>(s, g, batch, name);
   }
 }
 

@@ -326,7 +326,7 @@ const SmallVariant* pick_small(const GemmArgs& g, int epi, uint32_t cus, uint64_
 namespace prg {
 
 uint64_t gemm_small_cost(const GemmArgs& g, int epi, uint32_t cus) {
-  if (g.K % 256 != 0 || epi == kGemmSigmoidGate) return ~0ull;
+  if (g.K % 256 != 0) return ~0ull;
   uint64_t cost = 0;
   pick_small(g, epi, cus, &cost);
   return cost;

@@ -25,8 +25,9 @@ int ensure_prefill_ws(PrgModelState* st) {
     if (v >= 1) R = std::min<size_t>(R, static_cast<size_t>(v));
   }
   w.rows = static_cast<uint32_t>(R);
-  w.scores_elems = std::min<size_t>(static_cast<size_t>(kAttnQHeads) * R * align_up(st->max_seq, 64),
-                                    kPrefillScoresBytes / sizeof(uint16_t));
+  const size_t score_rows = static_cast<size_t>(kAttnQHeads) * R;
+  w.scores_elems = std::min<size_t>(score_rows * align_up(st->max_seq, 64), kPrefillScoresBytes / sizeof(uint16_t)) +
+                   score_rows * kAttnStatElems;
   const size_t bf = sizeof(uint16_t), f4 = sizeof(float);
   struct Item {
     void** slot;

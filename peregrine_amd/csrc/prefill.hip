@@ -1,14 +1,10 @@
-// Prompt-path (prefill) kernels other than the GEMMs: attention prepare and
-// softmax, the materialised causal attention driver, conv1d prefill with its
-// state publish, and the Gated DeltaNet prefill (q/k norms + gates, then the
+// Prompt-path (prefill) kernels other than the GEMMs and the attention itself
+// (attn_prefill.hip): attention prepare, conv1d prefill with its state publish, and the Gated DeltaNet prefill (q/k norms + gates, then the
 // token-sequential recurrence).
 //
 // Reference semantics (file:line in the reference tree):
 //   split_qg_many_bf16                       shaders/layout.metal:68-89
 //   qwen35_qk_norm_rope_append_many_bf16     shaders/attention.metal:146-220
-//   encodeMaterializedPrefillBf16            src/model/block_attn.zig:500-631
-//   prefill_softmax_scaled_masked_bf16       shaders/attention.metal:1463-1523
-//   sigmoid_mul_pair_inplace_bf16            shaders/elementwise.metal:88-99
 //   conv1d_silu_prefill_vec4_bf16 / _state   shaders/conv1d.metal:136-198
 //   qk_l2norm_prefill_bf16, gating_many_bf16 shaders/gated_norm.metal:191-268
 //   gated_delta_prefill_h128_norm_prepared_value_major_r8_bf16
@@ -17,7 +13,6 @@
 //                                            src/model/block_attn.zig:361-500
 #include "attention.hpp"
 #include "gdn.hpp"
-#include "gemm.hpp"
 #include "prefill.hpp"
 
 namespace {
@@ -25,70 +20,26 @@ namespace {
 using namespace prg;
 
 constexpr int kPrepThreads = 256;     // QWEN35_QK_PREPARE_THREADS (attention.metal:9)
-constexpr int kSoftmaxThreads = 256;  // PREFILL_SOFTMAX_THREADS (attention.metal:42)
-constexpr float kLog2e = 1.4426950408889634f;
 
-// Halving tree over blockDim.x == N threads in the reference's order
-// (partial[t] = op(partial[t], partial[t + stride]), stride N/2 .. 1). Every
-// thread gets the root. `sh` holds N floats. N == 256 combines the first two
-// levels from LDS in wave 0 and the rest inside that wave (v_permlane32_swap,
-// v_permlane16_swap, then DPP row shifts): the same pairs, so the same bits,
-// with two barriers instead of nine.
-template <bool MAX>
-__device__ inline float tree_op(float a, float b) {
-  return MAX ? fmaxf(a, b) : __fadd_rn(a, b);
-}
-template <bool MAX>
-__device__ inline float wave_tree_tail(float s) {  // strides 32 .. 1 within one wave; lane 0 holds the root
+// The last six levels (strides 32 .. 1) of the reference's halving tree within
+// one wave (v_permlane32_swap, v_permlane16_swap, then DPP row shifts): the
+// same pairs, so the same bits; lane 0 holds the root.
+__device__ inline float wave_tree_sum(float s) {
   {
     float x = s, y = s;
     swap32(x, y);
-    s = tree_op<MAX>(x, y);
+    s = __fadd_rn(x, y);
   }
   {
     float x = s, y = s;
     swap16(x, y);
-    s = tree_op<MAX>(x, y);
+    s = __fadd_rn(x, y);
   }
-  s = tree_op<MAX>(s, dpp_f<0x108>(s));  // row_shl:8 -- lane i with lane i + 8
-  s = tree_op<MAX>(s, dpp_f<0x104>(s));
-  s = tree_op<MAX>(s, dpp_f<0x102>(s));
-  s = tree_op<MAX>(s, dpp_f<0x101>(s));
+  s = __fadd_rn(s, dpp_f<0x108>(s));  // row_shl:8 -- lane i with lane i + 8
+  s = __fadd_rn(s, dpp_f<0x104>(s));
+  s = __fadd_rn(s, dpp_f<0x102>(s));
+  s = __fadd_rn(s, dpp_f<0x101>(s));
   return s;
-}
-template <int N, bool MAX>
-__device__ inline float tree_reduce(float v, float* sh) {
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  if constexpr (N == 256) {
-    if (threadIdx.x < kWave) {
-      const int l = threadIdx.x;
-      const float s = tree_op<MAX>(tree_op<MAX>(sh[l], sh[l + 128]), tree_op<MAX>(sh[l + 64], sh[l + 192]));
-      const float r = wave_tree_tail<MAX>(s);
-      if (l == 0) sh[N] = r;
-    }
-    __syncthreads();
-    return sh[N];
-  } else {
-#pragma unroll
-    for (int stride = N / 2; stride > 0; stride >>= 1) {
-      if (static_cast<int>(threadIdx.x) < stride)
-        sh[threadIdx.x] = tree_op<MAX>(sh[threadIdx.x], sh[threadIdx.x + stride]);
-      __syncthreads();
-    }
-    const float r = sh[0];
-    __syncthreads();
-    return r;
-  }
-}
-// `sh` holds N + 1 floats.
-template <int N>
-__device__ inline float tree_sum(float v, float* sh) {
-  return tree_reduce<N, false>(v, sh);
-}
-template <int N>
-__device__ inline float tree_max(float v, float* sh) {
-  return tree_reduce<N, true>(v, sh);
 }
 
 // ------------------------------------------------------- attention ----------
@@ -130,7 +81,7 @@ __global__ __launch_bounds__(kPrepThreads) void attn_prefill_prepare_kernel(
   }
   const float sq0 = __fmul_rn(x[0], x[0]), sq1 = __fmul_rn(x[1], x[1]);
   const float sq2 = __fmul_rn(x[2], x[2]), sq3 = __fmul_rn(x[3], x[3]);
-  const float root = wave_tree_tail<false>(__fadd_rn(__fadd_rn(sq0, sq2), __fadd_rn(sq1, sq3)));
+  const float root = wave_tree_sum(__fadd_rn(__fadd_rn(sq0, sq2), __fadd_rn(sq1, sq3)));
   const float ss = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, root), 0));
   const float scale = 1.0f / sqrtf(ss / static_cast<float>(kAttnHeadDim) + kAttnEps);
   uint16_t* dst = is_q ? q_out + static_cast<size_t>(lr) * kAttnHeadDim
@@ -150,64 +101,6 @@ __global__ __launch_bounds__(kPrepThreads) void attn_prefill_prepare_kernel(
   for (int i = 1; i < 4; ++i) {
     const uint32_t d = l + kWave * i;
     dst[d] = f2bf(__fmul_rn(__fmul_rn(x[i], scale), bf2f(w[d])));
-  }
-}
-
-// Causal softmax over one row of bf16 scores, in place (reference order: row
-// max of float(s)*scale over visible columns, then the sum of
-// exp2((v - max) * log2e), each thread striding the row, each reduced by a
-// halving tree). Row r of kv head z (rows z*4T .. ) is token r % T; column c is
-// visible iff c <= prefix + t. Columns [L, ld) are zeroed for the P*V GEMM.
-__global__ __launch_bounds__(kSoftmaxThreads) void attn_prefill_softmax_kernel(uint16_t* __restrict__ scores,
-                                                                               uint32_t ld, uint32_t L, uint32_t T,
-                                                                               uint32_t prefix, float scale) {
-  __shared__ float sh[kSoftmaxThreads + 1];
-  uint16_t* row = scores + static_cast<size_t>(blockIdx.x) * ld;
-  const uint32_t t = (blockIdx.x % (kAttnGroup * T)) % T;
-  const uint32_t vis = prefix + t;
-  // the P.V GEMM reads this row up to wend (zeros between vis and wend)
-  const uint32_t wend = causal_pv_columns(blockIdx.x % (kAttnGroup * T), T, prefix, L);
-  // The thread's first kCache columns (c = tid + 256 i) stay in registers
-  // across the three passes (one read of the row); later columns are read
-  // again. The arithmetic and its order per thread are unchanged. Masked
-  // columns (c > vis) are never read: the scores GEMM skips tiles that hold
-  // only masked columns, so they may hold anything.
-  constexpr int kCache = 8;
-  float xs[kCache];
-#pragma unroll
-  for (int i = 0; i < kCache; ++i) {
-    const uint32_t c = threadIdx.x + kSoftmaxThreads * i;
-    xs[i] = c <= vis ? __fmul_rn(bf2f(row[c]), scale) : 0.0f;
-  }
-  float m = -INFINITY;
-#pragma unroll
-  for (int i = 0; i < kCache; ++i) {
-    const uint32_t c = threadIdx.x + kSoftmaxThreads * i;
-    if (c < L) m = fmaxf(m, c > vis ? -INFINITY : xs[i]);
-  }
-  for (uint32_t c = threadIdx.x + kSoftmaxThreads * kCache; c <= vis; c += kSoftmaxThreads)
-    m = fmaxf(m, __fmul_rn(bf2f(row[c]), scale));
-  const float row_max = tree_max<kSoftmaxThreads>(m, sh);
-  float sum = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kCache; ++i) {
-    const uint32_t c = threadIdx.x + kSoftmaxThreads * i;
-    xs[i] = exp2f(__fmul_rn(__fsub_rn(xs[i], row_max), kLog2e));
-    if (c < L && c <= vis) sum += xs[i];
-  }
-  for (uint32_t c = threadIdx.x + kSoftmaxThreads * kCache; c <= vis; c += kSoftmaxThreads)
-    sum += exp2f(__fmul_rn(__fsub_rn(__fmul_rn(bf2f(row[c]), scale), row_max), kLog2e));
-  const float total = tree_sum<kSoftmaxThreads>(sum, sh);
-  const float denom = total == 0.0f ? 1.0f : total;
-#pragma unroll
-  for (int i = 0; i < kCache; ++i) {
-    const uint32_t c = threadIdx.x + kSoftmaxThreads * i;
-    if (c < wend) row[c] = c <= vis ? f2bf(xs[i] / denom) : uint16_t{0};
-  }
-  for (uint32_t c = threadIdx.x + kSoftmaxThreads * kCache; c < wend; c += kSoftmaxThreads) {
-    uint16_t p = 0;
-    if (c <= vis) p = f2bf(exp2f(__fmul_rn(__fsub_rn(__fmul_rn(bf2f(row[c]), scale), row_max), kLog2e)) / denom);
-    row[c] = p;
   }
 }
 
@@ -289,28 +182,11 @@ __global__ void conv1d_prefill_state_kernel(float* __restrict__ state, const uin
   }
 }
 
-// Sum of 128 values in tree_sum<128>'s order (entry i += entry i + stride
-// for stride 64, 32, ..., 1) within one wave: lane i holds entries i and
-// i + 64; the 32- and 16-lane steps pair lanes with v_permlane32_swap /
-// v_permlane16_swap, the rest shift within a DPP row. Returns the total to
-// every lane. Each step adds the same two values as the LDS tree, so the
-// bits are the tree's.
+// Sum of 128 values in the reference's halving tree's order (entry i += entry
+// i + stride for stride 64, 32, ..., 1) within one wave: lane i holds entries
+// i and i + 64. Returns the total to every lane.
 __device__ inline float tree128_wave(float lo, float hi) {
-  float s = __fadd_rn(lo, hi);
-  {
-    float x = s, y = s;
-    swap32(x, y);  // own value and lane i ^ 32's
-    s = __fadd_rn(x, y);
-  }
-  {
-    float x = s, y = s;
-    swap16(x, y);  // own value and the partner row's lane
-    s = __fadd_rn(x, y);
-  }
-  s = __fadd_rn(s, dpp_f<0x108>(s));  // row_shl:8 -- lane i += lane i + 8
-  s = __fadd_rn(s, dpp_f<0x104>(s));
-  s = __fadd_rn(s, dpp_f<0x102>(s));
-  s = __fadd_rn(s, dpp_f<0x101>(s));
+  const float s = wave_tree_sum(__fadd_rn(lo, hi));
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, s)));
 }
 
@@ -552,11 +428,6 @@ int launch_concat_rows(hipStream_t s, const uint16_t* a, const uint16_t* b, uint
   return PRG_OK;
 }
 
-size_t attn_prefill_scores_elems(uint32_t T, uint32_t prefix) {
-  const size_t L = static_cast<size_t>(prefix) + T, ld = (L + 63) / 64 * 64;
-  return static_cast<size_t>(kAttnQHeads) * T * ld;
-}
-
 int launch_attn_prefill_prepare(hipStream_t s, const uint16_t* qp, const uint16_t* q_w, const uint16_t* k_in,
                                 const uint16_t* k_w, const uint16_t* v_in, uint16_t* q_out, uint16_t* gate_out,
                                 uint16_t* cache_k, uint16_t* cache_v, uint32_t T, uint32_t start_rope,
@@ -566,57 +437,6 @@ int launch_attn_prefill_prepare(hipStream_t s, const uint16_t* qp, const uint16_
                      qp, q_w, k_in, k_w, v_in, q_out, gate_out, cache_k, cache_v, T, start_rope, start_cache, stride);
   PRG_CHECK_LAUNCH("attn_prefill_prepare");
   return PRG_OK;
-}
-
-int launch_attn_prefill(hipStream_t s, const uint16_t* q, const uint16_t* cache_k, const uint16_t* cache_v,
-                        const uint16_t* gate, uint16_t* out, uint16_t* scores, size_t scores_cap, uint32_t T,
-                        uint32_t prefix, uint32_t stride, float scale) {
-  // scores_cap: bf16 elements the score block holds
-  if (attn_prefill_scores_elems(T, prefix) > scores_cap)
-    return set_error(PRG_ERR_INVALID_ARG, "attention prefill: %u tokens after %u need %zu score elements, %zu held",
-                     T, prefix, attn_prefill_scores_elems(T, prefix), scores_cap);
-  const uint32_t L = prefix + T, ld = (L + 63) / 64 * 64;
-  const uint32_t rows = kAttnGroup * T;  // per kv head: q head in group x token
-  GemmArgs sc;
-  sc.a = q;
-  sc.lda = static_cast<uint64_t>(kAttnQHeads) * kAttnHeadDim;  // next token
-  sc.lda_hi = kAttnHeadDim;                                    // next q head of the group
-  sc.a_group = T;
-  sc.a_z = static_cast<uint64_t>(kAttnGroup) * kAttnHeadDim;
-  sc.b = cache_k;
-  sc.ldb = kAttnHeadDim;
-  sc.b_z = static_cast<uint64_t>(stride) * kAttnHeadDim;
-  sc.c = scores;
-  sc.ldc = ld;
-  sc.c_z = static_cast<uint64_t>(rows) * ld;
-  sc.M = rows;
-  sc.N = L;
-  sc.K = kAttnHeadDim;
-  sc.causal_T = T;
-  sc.causal_prefix = prefix;
-  if (int rc = launch_gemm_bf16(s, sc, kGemmStore, kAttnKvHeads, "attn_prefill.scores")) return rc;
-  hipLaunchKernelGGL(attn_prefill_softmax_kernel, dim3(kAttnKvHeads * rows), dim3(kSoftmaxThreads), 0, s, scores, ld,
-                     L, T, prefix, scale);
-  PRG_CHECK_LAUNCH("attn_prefill.softmax");
-  GemmArgs pv;
-  pv.a = scores;
-  pv.lda = ld;
-  pv.a_z = static_cast<uint64_t>(rows) * ld;
-  pv.b = cache_v;
-  pv.ldb = stride;
-  pv.b_z = static_cast<uint64_t>(kAttnHeadDim) * stride;
-  pv.c = out;
-  pv.res = gate;
-  pv.ldc = static_cast<uint64_t>(kAttnQHeads) * kAttnHeadDim;
-  pv.ldc_hi = kAttnHeadDim;
-  pv.c_group = T;
-  pv.c_z = static_cast<uint64_t>(kAttnGroup) * kAttnHeadDim;
-  pv.M = rows;
-  pv.N = kAttnHeadDim;
-  pv.K = L;
-  pv.causal_T = T;
-  pv.causal_prefix = prefix;
-  return launch_gemm_bf16(s, pv, kGemmSigmoidGate, kAttnKvHeads, "attn_prefill.values");
 }
 
 int launch_conv1d_prefill(hipStream_t s, float* state, const uint16_t* qkv, const uint16_t* w, uint16_t* out,

@@ -5,8 +5,11 @@
 
 namespace prg {
 
+// bf16 elements that a score row's statistics (two f32) take.
+constexpr size_t kAttnStatElems = 4;
 // Elements of the bf16 score workspace for T new tokens after `prefix` cached
-// ones: [kv head 4][q head in group 4 x T][round_up(prefix + T, 64)].
+// ones: [kv head 4][q head in group 4 x T][round_up(prefix + T, 64)], then two
+// f32 per row.
 size_t attn_prefill_scores_elems(uint32_t T, uint32_t prefix);
 
 // qp [T, 16, 512] (q ‖ gate per head), k_in/v_in [T, 4, 256] ->

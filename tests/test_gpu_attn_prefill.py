@@ -1,0 +1,40 @@
+"""Prefill attention against the oracle where its kernels change form: each
+split of the value dims (few, some and many tokens), each register window of
+the row statistics (contexts around 2048, 6144 and past 16384), contexts that
+end inside a 64-slot tile and inside a 16-byte chunk, and cache strides that
+are not a multiple of the tile. Cache slots past the context hold NaN. The
+bound is test_gpu_prefill's: one output ulp plus one flipped probability."""
+import numpy as np
+import pytest
+
+from peregrine_amd.synth import random_bf16
+from test_gpu_prefill import _check_attn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,prefix,stride", [(1, 0, 8), (33, 30, 64), (257, 3, 264), (513, 0, 520), (5, 2044, 2056),
+                                             (2, 6142, 6144), (3, 6150, 6400), (1, 16383, 16384), (2, 16400, 16448)])
+def test_attn_prefill_forms_vs_oracle(gpu, orc, T, prefix, stride):
+    from peregrine_amd import ops
+    from peregrine_amd.device import DeviceArray
+
+    print(f"[attn forms] T={T} prefix={prefix} stride={stride}", flush=True)
+    rng = np.random.default_rng(T * 7 + prefix)
+    L = prefix + T
+    q, gate = random_bf16(rng, (T, 4096)), random_bf16(rng, (T, 4096), std=2.0)
+    kc, vc = random_bf16(rng, (4, stride, 256)), random_bf16(rng, (4, 256, stride))
+    kc[:, L:] = 0x7FC0
+    vc[:, :, L:] = 0x7FC0
+    d = DeviceArray.from_numpy
+    guard = np.full((T + 1, 4096), 0x7FC1, np.uint16)
+    out = d(guard)
+    scores = DeviceArray((ops.attn_prefill_scores_bytes(T, prefix) // 2,), np.uint16)
+    ops.attn_prefill(d(q), d(kc), d(vc), d(gate), out, scores, T, prefix, stride)
+    gpu.synchronize()
+    got = out.numpy()
+    assert (got[T] == 0x7FC1).all()
+    vz = vc.copy()
+    vz[:, :, L:] = 0
+    ref = orc.sigmoid_mul_pair(orc.attn_prefill(q, kc, vz, T, prefix, stride), gate)
+    _check_attn(got[:T], ref, vz, f"attn prefill T={T} prefix={prefix}")
