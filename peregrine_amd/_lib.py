@@ -108,7 +108,9 @@ class _Lib:
 
     def __getattr__(self, name: str):
         if name.startswith("prg_"):
-            return getattr(self.load(), name)
+            fn = getattr(self.load(), name)
+            self.__dict__[name] = fn  # the next lookup finds it without this method
+            return fn
         raise AttributeError(name)
 
 
@@ -128,4 +130,6 @@ def check(fn_name: str, rc: int) -> None:
 
 
 def call(fn_name: str, *args) -> None:
-    check(fn_name, getattr(lib, fn_name)(*args))
+    rc = getattr(lib, fn_name)(*args)
+    if rc != 0:
+        check(fn_name, rc)
