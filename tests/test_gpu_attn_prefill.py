@@ -38,3 +38,29 @@ def test_attn_prefill_forms_vs_oracle(gpu, orc, T, prefix, stride):
     vz[:, :, L:] = 0
     ref = orc.sigmoid_mul_pair(orc.attn_prefill(q, kc, vz, T, prefix, stride), gate)
     _check_attn(got[:T], ref, vz, f"attn prefill T={T} prefix={prefix}")
+
+
+@pytest.mark.parametrize("T,start,stride", [(1, 0, 8), (63, 5, 72), (64, 0, 64), (65, 100, 168)])
+def test_prepare_aligned_equals_general(gpu, T, start, stride):
+    """16-byte aligned operands take the vector kernel, others the general one:
+    the same q, gate and cache bits (slots outside the call's stay untouched)."""
+    from peregrine_amd import ops
+    from peregrine_amd.device import DeviceArray
+
+    rng = np.random.default_rng(T)
+    ins = [random_bf16(rng, (n,), std=std, mean=mean) for n, std, mean in
+           [(T * 8192, 2.0, 0.0), (256, 0.1, 1.0), (T * 1024, 2.0, 0.0), (256, 0.1, 1.0), (T * 1024, 1.0, 0.0)]]
+    sizes = [T * 4096, T * 4096, 4 * stride * 256, 4 * 256 * stride]
+
+    def run(shift):  # operands `shift` values past a 16-byte boundary
+        def dev(a):
+            return DeviceArray.from_numpy(np.concatenate([np.zeros(shift, np.uint16), a, np.zeros(8, np.uint16)]))
+
+        arrays = [dev(a) for a in ins] + [dev(np.full(n, 0x7FC1, np.uint16)) for n in sizes]
+        p = [a.ptr + 2 * shift for a in arrays]
+        ops.attn_prefill_prepare(*p, T, start, start, stride)
+        gpu.synchronize()
+        return [a.numpy()[shift:shift + n] for a, n in zip(arrays[5:], sizes)]
+
+    for a, b, what in zip(run(0), run(1), ("q", "gate", "K cache", "V cache")):
+        np.testing.assert_array_equal(a, b, err_msg=what)
