@@ -213,8 +213,10 @@ __device__ inline float2 conv_src(const float* state, const uint16_t* qkv, uint3
 __device__ inline float conv_tap(float acc, float w, float x) { return __fadd_rn(acc, __fmul_rn(w, x)); }
 
 // Thread = (channel pair, 16-token chunk): out[t, c] = bf16(silu(sum_j w[c, j] * x(t + j))).
-__global__ __launch_bounds__(256) void conv1d_prefill_kernel(const float* __restrict__ state,
-                                                             const uint16_t* __restrict__ qkv,
+// The first chunk's threads are the only ones that read the old state, so they
+// also leave the new one behind, state[j, c] = x(T + j), once they have read it
+// (a launch of its own for that took 4.7 us).
+__global__ __launch_bounds__(256) void conv1d_prefill_kernel(float* state, const uint16_t* __restrict__ qkv,
                                                              const uint16_t* __restrict__ w,
                                                              uint16_t* __restrict__ out, uint32_t T,
                                                              uint32_t has_state) {
@@ -227,6 +229,16 @@ __global__ __launch_bounds__(256) void conv1d_prefill_kernel(const float* __rest
   const float w1[4] = {bf_lo(wv.z), bf_hi(wv.z), bf_lo(wv.w), bf_hi(wv.w)};
   const bool hs = has_state != 0;
   const uint32_t t1 = min(t0 + kConvChunk, T);
+  float2 next[kGdnConvK - 1];  // the last three entries of the virtual sequence
+  if (t0 == 0)
+    for (uint32_t j = 0; j < kGdnConvK - 1; ++j) next[j] = conv_src(state, qkv, T + j, c, hs);
+  auto publish = [&]() {
+    if (t0 != 0) return;
+    for (uint32_t j = 0; j < kGdnConvK - 1; ++j) {
+      state[j * kGdnConvDim + c] = next[j].x;
+      state[j * kGdnConvDim + c + 1] = next[j].y;
+    }
+  };
   if (t1 - t0 == kConvChunk) {
     // A full chunk issues all of its kConvChunk + 3 loads before the first
     // tap (the same arithmetic per output as the loop below).
@@ -242,6 +254,7 @@ __global__ __launch_bounds__(256) void conv1d_prefill_kernel(const float* __rest
                          (static_cast<uint32_t>(f2bf(a1 / (1.0f + expf(-a1)))) << 16);
       *reinterpret_cast<uint32_t*>(out + static_cast<size_t>(t0 + i) * kGdnConvDim + c) = o;
     }
+    publish();
     return;
   }
   float2 h0 = conv_src(state, qkv, t0, c, hs), h1 = conv_src(state, qkv, t0 + 1, c, hs),
@@ -258,21 +271,7 @@ __global__ __launch_bounds__(256) void conv1d_prefill_kernel(const float* __rest
     h1 = h2;
     h2 = h3;
   }
-}
-
-// state[j, c] = x(T + j): the last three entries of the virtual sequence.
-// Runs after conv1d_prefill_kernel (which reads the old state).
-__global__ void conv1d_prefill_state_kernel(float* __restrict__ state, const uint16_t* __restrict__ qkv, uint32_t T,
-                                            uint32_t has_state) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= kGdnConvDim) return;
-  for (uint32_t j = 0; j < kGdnConvK - 1; ++j) {
-    const uint32_t u = T + j;  // u > j: state[u] is read before it is rewritten
-    float x = 0.0f;
-    if (u < kGdnConvK - 1) x = has_state ? state[u * kGdnConvDim + c] : 0.0f;
-    else x = bf2f(qkv[static_cast<size_t>(u - (kGdnConvK - 1)) * kGdnConvDim + c]);
-    state[j * kGdnConvDim + c] = x;
-  }
+  publish();
 }
 
 // Sum of 128 values in the reference's halving tree's order (entry i += entry
@@ -550,8 +549,6 @@ int launch_conv1d_prefill(hipStream_t s, float* state, const uint16_t* qkv, cons
   hipLaunchKernelGGL(conv1d_prefill_kernel, dim3(static_cast<uint32_t>((threads + 255) / 256)), dim3(256), 0, s, state,
                      qkv, w, out, T, has_state);
   PRG_CHECK_LAUNCH("conv1d_prefill");
-  hipLaunchKernelGGL(conv1d_prefill_state_kernel, dim3(kGdnConvDim / 256), dim3(256), 0, s, state, qkv, T, has_state);
-  PRG_CHECK_LAUNCH("conv1d_prefill_state");
   return PRG_OK;
 }
 
