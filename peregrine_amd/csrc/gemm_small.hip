@@ -295,14 +295,14 @@ int launch_small_rows(hipStream_t s, const GemmArgs& g, int mw, const char* name
 
 // Cost of a round of blocks in units of gemm_q4_kernel rows (0.255 us at
 // K = 4096), from launches timed alone over rotating weights: 16 / 32 / 64 /
-// 128 weight rows per block take 13 / 14 / 20 / 33 us with up to 64 activation
-// rows and 20.5 / 20.5 / 34 / 44.5 us with up to 128.
+// 128 weight rows per block take 13 / 14 / 20 / 34 us with up to 64 activation
+// rows and 14.4 / 20 / 35 / 46 us with up to 128.
 struct SmallVariant {
   int tn, mw;
   uint32_t cost;
 };
 constexpr SmallVariant kSmallVariants[] = {{1, 1, 51}, {2, 1, 55},  {4, 1, 75},  {8, 1, 130},
-                                           {1, 2, 80}, {2, 2, 80}, {4, 2, 133}, {8, 2, 175}};
+                                           {1, 2, 56}, {2, 2, 80}, {4, 2, 133}, {8, 2, 175}};
 
 const SmallVariant* pick_small(const GemmArgs& g, int epi, uint32_t cus, uint64_t* cost) {
   const SmallVariant* best = nullptr;
