@@ -35,7 +35,9 @@ __device__ inline uint32_t clamp_bytes(uint64_t n) { return n < 0xffffffffull ? 
 // last visible slot are skipped. K is the A operand, so a lane holds four
 // consecutive columns of one row; they leave through a wave's own LDS rows as
 // 128-byte row segments. Same products and k order per score as a 16x16x32
-// tiling with the operands exchanged.
+// tiling with the operands exchanged. Bound by the score writes (2.8 TB/s at a
+// long context; matrix cores 30% busy). 1600 tokens 47 -> 25 us, 1021 tokens
+// after 15003 357 -> 180-196 us (a 128 x 128 GEMM before).
 __global__ __launch_bounds__(256) void attn_prefill_scores_kernel(const uint16_t* __restrict__ q,
                                                                   const uint16_t* __restrict__ cache_k,
                                                                   uint16_t* __restrict__ scores, uint32_t T,
@@ -152,8 +154,11 @@ __device__ inline float prob_exp(float x, float m) {
 // 256 n + 4 l .. +3, i.e. the reference's 256 strided partial sums 4 l .. 4 l + 3
 // (each summed in column order), which then combine in its halving tree's
 // pairs: t with t + 128 is lane l with l + 32, t + 64 lane l + 16, and so on
-// down to the lane's own four. The first NG groups stay in registers between
-// the two passes; later ones are read again.
+// down to the lane's own four. The first NG groups stay in registers (packed:
+// their f32 values took 256 registers and a wave per SIMD, 260 us) between the
+// two passes; later ones are read again. Bound by reading the scores once
+// (3.2 TB/s). 1600 tokens 16 us, 1021 after 15003 160-179 us, where the softmax
+// that rewrote the row took 49 and 727 us.
 template <int NG>
 __global__ __launch_bounds__(256) void attn_prefill_stats_kernel(const uint16_t* __restrict__ scores,
                                                                  float2* __restrict__ stats, uint32_t ld, uint32_t T,
@@ -233,7 +238,10 @@ __global__ __launch_bounds__(256) void attn_prefill_stats_kernel(const uint16_t*
 // them to LDS; four consumer waves (2 x 32 rows, 2 x half of the dims) copy the V
 // tiles straight to LDS kBufs - 1 tiles ahead and run the matrix instructions,
 // in slot order from 0, so a row's bits do not depend on the chunk it is
-// computed in.
+// computed in. Per tile a producer wave's ~240 VALU operations, the LDS traffic
+// (120 KB) and the matrix instructions (a quarter of the time) meet at one
+// barrier. 1600 tokens 57 -> 46 us, 1021 after 15003 323 -> 245-290 us (a GEMM
+// over stored probabilities before).
 template <int DS>
 __global__ __launch_bounds__(kPvThreads) void attn_prefill_pv_kernel(const uint16_t* __restrict__ scores,
                                                                      const float2* __restrict__ stats,

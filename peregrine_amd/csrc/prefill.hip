@@ -406,7 +406,8 @@ __global__ __launch_bounds__(256) void gdn_prefill_kernel(float* __restrict__ st
       if (tid < kGdnChunk) sgk[buf][tid] = make_float4(rg, rbt, rkq, 0.f);
     } else {
       // k.q of the chunk's tokens, four per 32 lanes (each lane its float4 of
-      // both): a quarter of an operation per token instead of 13 in the loop.
+      // both): a few operations per chunk instead of 13 per token in the loop
+      // (1600 tokens: 292 -> 267 us).
       if (tid < kGdnChunk) *reinterpret_cast<float2*>(&sgk[buf][tid]) = make_float2(rg, rbt);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
