@@ -131,6 +131,11 @@ __global__ __launch_bounds__(256) void attn_prefill_scores_kernel(const uint16_t
             make_uint2(pack_bf16(acc[x][j][0], acc[x][j][1]), pack_bf16(acc[x][j][2], acc[x][j][3]));
       }
     PRG_WAIT_VMCNT(0);  // the next tile has landed (and the previous tile's stores)
+    // The wave's lanes exchange the tile through its own rows of sS: in order in
+    // the LDS pipe, and kept so by the compiler.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint32_t r = 8 * i + (lane >> 3), ch = lane & 7;

@@ -40,6 +40,30 @@ def test_attn_prefill_forms_vs_oracle(gpu, orc, T, prefix, stride):
     _check_attn(got[:T], ref, vz, f"attn prefill T={T} prefix={prefix}")
 
 
+@pytest.mark.parametrize("T,prefix", [(513, 3000), (1600, 0), (1021, 15003)])
+def test_attn_prefill_long_segments_vs_oracle(gpu, orc, T, prefix):
+    """Score blocks that walk 3, 4 and 16 tiles, so that each K buffer is used
+    again. Sampled rows: the oracle's row t of T tokens is its only row of one
+    token after prefix + t."""
+    from peregrine_amd import ops
+    from peregrine_amd.device import DeviceArray
+
+    print(f"[attn segments] T={T} prefix={prefix}", flush=True)
+    rng = np.random.default_rng(T + prefix)
+    stride = (prefix + T + 63) // 64 * 64
+    q, gate = random_bf16(rng, (T, 4096)), random_bf16(rng, (T, 4096), std=2.0)
+    kc, vc = random_bf16(rng, (4, stride, 256)), random_bf16(rng, (4, 256, stride))
+    d = DeviceArray.from_numpy
+    out = DeviceArray((T, 4096), np.uint16)
+    scores = DeviceArray((ops.attn_prefill_scores_bytes(T, prefix) // 2,), np.uint16)
+    ops.attn_prefill(d(q), d(kc), d(vc), d(gate), out, scores, T, prefix, stride)
+    gpu.synchronize()
+    rows = np.unique([0, 31, 32, T // 2, T - 33, T - 1])
+    ref = np.concatenate([orc.sigmoid_mul_pair(orc.attn_prefill(q[t:t + 1], kc, vc, 1, prefix + int(t), stride),
+                                               gate[t:t + 1]) for t in rows])
+    _check_attn(out.numpy()[rows], ref, vc, f"attn prefill T={T} prefix={prefix}")
+
+
 @pytest.mark.parametrize("T,start,stride", [(1, 0, 8), (63, 5, 72), (64, 0, 64), (65, 100, 168)])
 def test_prepare_aligned_equals_general(gpu, T, start, stride):
     """16-byte aligned operands take the vector kernel, others the general one:
