@@ -6,6 +6,8 @@ Every call goes straight to libperegrine_hip.so; there is no CPU fallback.
 """
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 
 from ._lib import call
@@ -16,7 +18,11 @@ QMV_FAST_RESULTS_PER_THREADGROUP = 8  # linear_q4.zig:11 (partial = 8 rows)
 
 
 def _s(stream):
-    return stream if stream else None
+    """Stream handle: an int, 0 or None. c_void_p refuses anything else, which
+    the bound argument type would not (a str passes there as its address)."""
+    if not stream or type(stream) is int:
+        return stream or None
+    return C.c_void_p(stream)
 
 
 def _dev(x):
