@@ -417,6 +417,15 @@ int prg_q4_qmm_silu_gate_bf16(void *stream, const uint16_t *x, const uint32_t *g
                               const uint16_t *up_biases, uint16_t *out, uint32_t token_count,
                               uint32_t out_dim, uint32_t in_dim);
 
+/* Which kernel a prompt GEMM of these sizes takes on the current device (host
+ * arithmetic, no launch): 10 t + m = few-row form of 16 t weight and 64 m
+ * activation rows per block, 192 / 256 = row tile of the kernel that
+ * dequantises on the way to LDS, 1256 / 1320 = row tile of the one that copies
+ * prepared weights, 0 = sizes refused. epilogue: 0 store, 1 residual add, 2 SiLU
+ * gate (out_dims then holds gate and up). All give the same bits. */
+int prg_q4_qmm_route(uint32_t epilogue, uint32_t token_count, const uint32_t *out_dims, uint32_t weights,
+                     uint32_t in_dim, uint32_t prepared);
+
 /* For T tokens: split packed q [T, 16, 512] into q_output/gate_output
  * [T, 16, 256]; RMSNorm + RoPE (positions start_rope_pos + t) of q and of
  * k_input [T, 4, 256] (normed value kept in f32 through RoPE); append K/V at

@@ -487,6 +487,14 @@ inline int dma_override() {
   return atoi(e);
 }
 
+// Column tiles of gemm_dma_kernel: 128 outputs of the pair, 256 of a store segment.
+inline uint32_t dma_tiles_n(const GemmArgs& g, int epi) {
+  if (epi == kGemmSiluPair) return (g.q[0].n + 127) / 128;
+  uint32_t tiles = 0;
+  for (uint32_t i = 0; i < g.nq; ++i) tiles += (g.q[i].n + 255) / 256;
+  return tiles;
+}
+
 // g: as launch_gemm_q4 leaves it (segments' tile0 in 128-column tiles).
 template <int EPI, int BM>
 int launch_dma(hipStream_t s, GemmArgs g, uint32_t tiles_n, const char* name) {
@@ -507,43 +515,58 @@ int launch_dma(hipStream_t s, GemmArgs g, uint32_t tiles_n, const char* name) {
   return PRG_OK;
 }
 
+// The kernel a launch takes: gemm_dma_kernel with `dma` rows per tile, or the
+// few-row form `small`, or gemm_q4_kernel with `bm` rows per tile.
+struct Q4Route {
+  uint32_t dma = 0, bm = 0;
+  GemmSmallPick small;
+};
+
+// g: as launch_gemm_q4 leaves it. Every launch looks once at
+// PEREGRINE_GEMM_DMA and once through the few-row forms.
+Q4Route route_q4(const GemmArgs& g, int epi) {
+  const bool pair = epi == kGemmSiluPair;
+  const uint32_t cus = gemm_device_cus();
+  const uint32_t tiles_n = pair ? (g.q[0].n + 63) / 64 : g.q[g.nq - 1].tile0 + (g.q[g.nq - 1].n + 127) / 128;
+  auto cost = [&](uint32_t bm, uint32_t tiles, uint64_t round) -> uint64_t {
+    const uint32_t blocks = ((g.M + bm - 1) / bm) * tiles;
+    return static_cast<uint64_t>((blocks + cus - 1) / cus) * round;
+  };
+  const uint64_t c192 = cost(192, tiles_n, 192), cq256 = cost(256, tiles_n, 256), cold = std::min(c192, cq256);
+  const int force = dma_override();
+  Q4Route r;
+  // Few rows: where blocks of 16 to 128 weight rows take fewer units than the
+  // best of the row-tiled kernels (a PEREGRINE_GEMM_DMA override keeps those).
+  if (force < 0) r.small = gemm_small_pick(g, epi, cus);
+  if (epi != kGemmResidual) {
+    bool dense = true;
+    for (uint32_t i = 0; i < g.nq; ++i) dense = dense && g.q[i].dense != nullptr;
+    if (dense) {
+      const uint32_t tiles_nd = dma_tiles_n(g, epi);
+      const uint64_t c256 = cost(256, tiles_nd, kDmaRoundCost256), c320 = cost(320, tiles_nd, kDmaRoundCost320);
+      if (force == 256 || force == 320) {
+        r.dma = static_cast<uint32_t>(force);
+      } else if (force < 0 && std::min(c256, c320) < std::min(cold, r.small.cost)) {
+        r.dma = c320 < c256 ? 320 : 256;
+      }
+    }
+  }
+  if (r.dma || r.small.cost >= cold) r.small = GemmSmallPick{};
+  r.bm = c192 < cq256 ? 192 : 256;
+  return r;
+}
+
 template <int EPI>
 int launch_q4_t(hipStream_t s, const GemmArgs& g, const char* name) {
   const uint32_t tiles_n = (EPI == kGemmSiluPair) ? (g.q[0].n + 63) / 64
                                                   : g.q[g.nq - 1].tile0 + (g.q[g.nq - 1].n + 127) / 128;
-  const uint32_t cus = gemm_device_cus();
-  auto cost = [&](uint32_t bm) -> uint64_t {
-    const uint32_t blocks = ((g.M + bm - 1) / bm) * tiles_n;
-    return static_cast<uint64_t>((blocks + cus - 1) / cus) * bm;
-  };
-  const uint64_t cold = std::min(cost(192), cost(256));
-  // Few rows: where blocks of 16 to 128 weight rows take fewer units than the
-  // best of the row-tiled kernels (a PEREGRINE_GEMM_DMA override keeps those).
-  const uint64_t small = dma_override() < 0 ? gemm_small_cost(g, EPI, cus) : ~0ull;
-  if constexpr (EPI == kGemmSiluPair || EPI == kGemmStore) {
-    bool dense = true;
-    for (uint32_t i = 0; i < g.nq; ++i) dense = dense && g.q[i].dense != nullptr;
-    if (dense) {
-      // columns per block: 128 outputs of the pair, 256 of a store segment
-      uint32_t tiles_nd = 0;
-      if constexpr (EPI == kGemmSiluPair) {
-        tiles_nd = (g.q[0].n + 127) / 128;
-      } else {
-        for (uint32_t i = 0; i < g.nq; ++i) tiles_nd += (g.q[i].n + 255) / 256;
-      }
-      auto cost_dma = [&](uint32_t bm, uint64_t round) -> uint64_t {
-        const uint32_t blocks = ((g.M + bm - 1) / bm) * tiles_nd;
-        return static_cast<uint64_t>((blocks + cus - 1) / cus) * round;
-      };
-      const uint64_t c256 = cost_dma(256, kDmaRoundCost256), c320 = cost_dma(320, kDmaRoundCost320);
-      int pick = dma_override();
-      if (pick < 0) pick = std::min(c256, c320) < std::min(cold, small) ? (c320 < c256 ? 320 : 256) : 0;
-      if (pick == 320) return launch_dma<EPI, 320>(s, g, tiles_nd, name);
-      if (pick == 256) return launch_dma<EPI, 256>(s, g, tiles_nd, name);
-    }
+  const Q4Route r = route_q4(g, EPI);
+  if constexpr (EPI != kGemmResidual) {
+    if (r.dma == 320) return launch_dma<EPI, 320>(s, g, dma_tiles_n(g, EPI), name);
+    if (r.dma == 256) return launch_dma<EPI, 256>(s, g, dma_tiles_n(g, EPI), name);
   }
-  if (small < cold) return launch_gemm_small(s, g, EPI, cus, name);
-  if (cost(192) < cost(256)) return launch_q4_bm<EPI, 192>(s, g, tiles_n, name);
+  if (r.small.tn) return launch_gemm_small(s, g, EPI, r.small, name);
+  if (r.bm == 192) return launch_q4_bm<EPI, 192>(s, g, tiles_n, name);
   return launch_q4_bm<EPI, 256>(s, g, tiles_n, name);
 }
 
@@ -679,6 +702,26 @@ int prg_q4_qmm_silu_gate_bf16(void* stream, const uint16_t* x, const uint32_t* g
   g.M = token_count;
   g.K = in_dim;
   return launch_gemm_q4(as_stream(stream), g, kGemmSiluPair, "prg_q4_qmm_silu_gate_bf16");
+}
+
+int prg_q4_qmm_route(uint32_t epilogue, uint32_t token_count, const uint32_t* out_dims, uint32_t weights,
+                     uint32_t in_dim, uint32_t prepared) {
+  if (!out_dims || weights < 1 || weights > kGemmMaxSegs || epilogue > kGemmSiluPair || token_count == 0) return 0;
+  GemmArgs g;
+  uint32_t tile = 0;
+  for (uint32_t i = 0; i < weights; ++i) {
+    if (out_dims[i] == 0) return 0;
+    g.q[i].n = out_dims[i];
+    g.q[i].tile0 = tile;
+    g.q[i].dense = prepared ? reinterpret_cast<uint16_t*>(16) : nullptr;  // tested for null only
+    tile += (out_dims[i] + kBN - 1) / kBN;
+  }
+  g.nq = weights;
+  g.M = token_count;
+  g.K = in_dim;
+  const Q4Route r = route_q4(g, static_cast<int>(epilogue));
+  if (r.dma) return static_cast<int>(1000 + r.dma);
+  return r.small.tn ? 10 * r.small.tn + r.small.mw : static_cast<int>(r.bm);
 }
 
 }  // extern "C"

@@ -53,11 +53,16 @@ struct GemmArgs {
 // Q4 weights in g.q[0..nq). K % 64 == 0; A rows 16-byte aligned (lda % 8 == 0).
 // The residual epilogue reads g.res [M, q[0].n].
 int launch_gemm_q4(hipStream_t s, GemmArgs g, int epi, const char* name);
-// Few activation rows (gemm_small.hip): the launch's cost on `cus` CUs in units
-// of gemm_q4_kernel rows (~0 when the kernel does not take it), and the launch;
-// g as launch_gemm_q4 has checked it.
-uint64_t gemm_small_cost(const GemmArgs& g, int epi, uint32_t cus);
-int launch_gemm_small(hipStream_t s, const GemmArgs& g, int epi, uint32_t cus, const char* name);
+// Few activation rows (gemm_small.hip): the form that takes a launch in the
+// least time on `cus` CUs and its cost in units of gemm_q4_kernel rows (tn 0 and
+// ~0 when the kernel does not take it), and the launch of that form; g as
+// launch_gemm_q4 has checked it.
+struct GemmSmallPick {
+  int tn = 0, mw = 0;  // 16-row weight tiles, 64-row activation tiles per block
+  uint64_t cost = ~0ull;
+};
+GemmSmallPick gemm_small_pick(const GemmArgs& g, int epi, uint32_t cus);
+int launch_gemm_small(hipStream_t s, const GemmArgs& g, int epi, const GemmSmallPick& pick, const char* name);
 // Prepared bf16 copy out [n, K] of Q4 weights (w, sc, bi): the values the Q4
 // GEMM dequantises per tile.
 int launch_dequant_dense(hipStream_t s, const uint32_t* w, const uint16_t* sc, const uint16_t* bi, uint16_t* out,

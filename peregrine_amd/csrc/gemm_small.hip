@@ -304,8 +304,13 @@ struct SmallVariant {
 constexpr SmallVariant kSmallVariants[] = {{1, 1, 51}, {2, 1, 55},  {4, 1, 75},  {8, 1, 130},
                                            {1, 2, 56}, {2, 2, 80}, {4, 2, 133}, {8, 2, 175}};
 
-const SmallVariant* pick_small(const GemmArgs& g, int epi, uint32_t cus, uint64_t* cost) {
-  const SmallVariant* best = nullptr;
+}  // namespace
+
+namespace prg {
+
+GemmSmallPick gemm_small_pick(const GemmArgs& g, int epi, uint32_t cus) {
+  GemmSmallPick best;
+  if (g.K % 256 != 0) return best;
   for (const SmallVariant& v : kSmallVariants) {
     if (epi == kGemmSiluPair ? v.tn < 4 : v.tn > 4) continue;
     const uint32_t cols = 16 * (epi == kGemmSiluPair ? v.tn / 2 : v.tn), rows = 64 * v.mw;
@@ -313,40 +318,24 @@ const SmallVariant* pick_small(const GemmArgs& g, int epi, uint32_t cus, uint64_
     for (uint32_t i = 0; i < (epi == kGemmSiluPair ? 1 : g.nq); ++i) blocks += (g.q[i].n + cols - 1) / cols;
     blocks *= (g.M + rows - 1) / rows;
     const uint64_t c = (blocks + cus - 1) / cus * v.cost;
-    if (!best || c < *cost) {
-      best = &v;
-      *cost = c;
-    }
+    if (c < best.cost) best = {v.tn, v.mw, c};
   }
   return best;
 }
 
-}  // namespace
-
-namespace prg {
-
-uint64_t gemm_small_cost(const GemmArgs& g, int epi, uint32_t cus) {
-  if (g.K % 256 != 0) return ~0ull;
-  uint64_t cost = 0;
-  pick_small(g, epi, cus, &cost);
-  return cost;
-}
-
-int launch_gemm_small(hipStream_t s, const GemmArgs& g, int epi, uint32_t cus, const char* name) {
-  uint64_t cost = 0;
-  const SmallVariant* v = pick_small(g, epi, cus, &cost);
+int launch_gemm_small(hipStream_t s, const GemmArgs& g, int epi, const GemmSmallPick& v, const char* name) {
   if (epi == kGemmSiluPair) {
-    if (v->tn == 4) return launch_small_rows<kGemmSiluPair, 4>(s, g, v->mw, name);
-    return launch_small_rows<kGemmSiluPair, 8>(s, g, v->mw, name);
+    if (v.tn == 4) return launch_small_rows<kGemmSiluPair, 4>(s, g, v.mw, name);
+    return launch_small_rows<kGemmSiluPair, 8>(s, g, v.mw, name);
   }
   if (epi == kGemmResidual) {
-    if (v->tn == 1) return launch_small_rows<kGemmResidual, 1>(s, g, v->mw, name);
-    if (v->tn == 2) return launch_small_rows<kGemmResidual, 2>(s, g, v->mw, name);
-    return launch_small_rows<kGemmResidual, 4>(s, g, v->mw, name);
+    if (v.tn == 1) return launch_small_rows<kGemmResidual, 1>(s, g, v.mw, name);
+    if (v.tn == 2) return launch_small_rows<kGemmResidual, 2>(s, g, v.mw, name);
+    return launch_small_rows<kGemmResidual, 4>(s, g, v.mw, name);
   }
-  if (v->tn == 1) return launch_small_rows<kGemmStore, 1>(s, g, v->mw, name);
-  if (v->tn == 2) return launch_small_rows<kGemmStore, 2>(s, g, v->mw, name);
-  return launch_small_rows<kGemmStore, 4>(s, g, v->mw, name);
+  if (v.tn == 1) return launch_small_rows<kGemmStore, 1>(s, g, v.mw, name);
+  if (v.tn == 2) return launch_small_rows<kGemmStore, 2>(s, g, v.mw, name);
+  return launch_small_rows<kGemmStore, 4>(s, g, v.mw, name);
 }
 
 }  // namespace prg

@@ -100,3 +100,18 @@ def qwen35_config(hidden=4096, intermediate=12288, layers=32, vocab=248320, bits
     tc.update(text_overrides)
     return {"model_type": "qwen3_5", "text_config": tc,
             "quantization": {"group_size": group, "bits": bits, "mode": mode}}
+
+
+# --------------------------------------------------------------- prompt GEMM ---
+STORE, RESIDUAL, PAIR = 0, 1, 2
+
+
+def qmm_route(epilogue: int, rows: int, out_dims, in_dim: int, prepared: bool = False) -> int:
+    """prg_q4_qmm_route: 10 t + m few-row form, 192 / 256 and 1256 / 1320 the
+    row-tiled kernels, 0 sizes refused. out_dims: one int per weight."""
+    import ctypes as C
+
+    from peregrine_amd._lib import lib
+
+    dims = (C.c_uint32 * len(out_dims))(*out_dims)
+    return lib.prg_q4_qmm_route(epilogue, rows, C.addressof(dims), len(out_dims), in_dim, int(prepared))
