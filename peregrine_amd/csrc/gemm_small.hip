@@ -294,15 +294,19 @@ int launch_small_rows(hipStream_t s, const GemmArgs& g, int mw, const char* name
 }
 
 // Cost of a round of blocks in units of gemm_q4_kernel rows (0.255 us at
-// K = 4096), from launches timed alone over rotating weights: 16 / 32 / 64 /
-// 128 weight rows per block take 13 / 14 / 20 / 34 us with up to 64 activation
-// rows and 14.4 / 20 / 35 / 46 us with up to 128.
+// K = 4096), from launches of 192 to 256 blocks over rotating weights: with up to
+// 64 activation rows 16 / 32 / 64 / 128 weight rows per block take 13 / 14 / 20 /
+// 34 us; with up to 128, 18.4 / 20 / 35 / 46 us. {1, 2} and {2, 2} are the pick
+// only where the column tiles leave the others a nearly empty round: 384 rows x
+// 1360 outputs 18.4 us against 20.9 of {4, 1}, 322 x 2720 20.1 against 26.4 of
+// {4, 2}. A pair form {4, 2} gained nothing on two rounds of {4, 1} (322 x 2720:
+// 13.5 against 12.6 us at K = 1024, 35.0 / 34.0 at 4096, 90.6 / 90.9 at 12288).
 struct SmallVariant {
   int tn, mw;
   uint32_t cost;
 };
-constexpr SmallVariant kSmallVariants[] = {{1, 1, 51}, {2, 1, 55},  {4, 1, 75},  {8, 1, 130},
-                                           {1, 2, 56}, {2, 2, 80}, {4, 2, 133}, {8, 2, 175}};
+constexpr SmallVariant kSmallPlain[] = {{1, 1, 51}, {2, 1, 55}, {4, 1, 75}, {1, 2, 72}, {2, 2, 80}, {4, 2, 133}};
+constexpr SmallVariant kSmallPair[] = {{4, 1, 75}, {8, 1, 130}, {8, 2, 175}};
 
 }  // namespace
 
@@ -311,21 +315,25 @@ namespace prg {
 GemmSmallPick gemm_small_pick(const GemmArgs& g, int epi, uint32_t cus) {
   GemmSmallPick best;
   if (g.K % 256 != 0) return best;
-  for (const SmallVariant& v : kSmallVariants) {
-    if (epi == kGemmSiluPair ? v.tn < 4 : v.tn > 4) continue;
-    const uint32_t cols = 16 * (epi == kGemmSiluPair ? v.tn / 2 : v.tn), rows = 64 * v.mw;
+  const bool pair = epi == kGemmSiluPair;
+  auto consider = [&](const SmallVariant& v) {
+    const uint32_t cols = 16 * (pair ? v.tn / 2 : v.tn), rows = 64 * v.mw;
     uint64_t blocks = 0;
-    for (uint32_t i = 0; i < (epi == kGemmSiluPair ? 1 : g.nq); ++i) blocks += (g.q[i].n + cols - 1) / cols;
+    for (uint32_t i = 0; i < (pair ? 1 : g.nq); ++i) blocks += (g.q[i].n + cols - 1) / cols;
     blocks *= (g.M + rows - 1) / rows;
     const uint64_t c = (blocks + cus - 1) / cus * v.cost;
     if (c < best.cost) best = {v.tn, v.mw, c};
-  }
+  };
+  if (pair)
+    for (const SmallVariant& v : kSmallPair) consider(v);
+  else
+    for (const SmallVariant& v : kSmallPlain) consider(v);
   return best;
 }
 
 int launch_gemm_small(hipStream_t s, const GemmArgs& g, int epi, const GemmSmallPick& v, const char* name) {
   if (epi == kGemmSiluPair) {
-    if (v.tn == 4) return launch_small_rows<kGemmSiluPair, 4>(s, g, v.mw, name);
+    if (v.tn == 4) return launch_small<kGemmSiluPair, 4, 1, 128, 8, 3>(s, g, name);
     return launch_small_rows<kGemmSiluPair, 8>(s, g, v.mw, name);
   }
   if (epi == kGemmResidual) {

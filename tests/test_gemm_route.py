@@ -26,6 +26,16 @@ def test_model_widths(rows, routes):
     assert got == routes
 
 
+# where the column tiles leave the 32- and 64-row forms a nearly empty round; the two-round launch of
+# 16 x 128 rows costs more than one of 64 x 128
+@pytest.mark.parametrize("epilogue,rows,outs,route", [
+    (STORE, 384, 1360, 12), (STORE, 640, 816, 12), (STORE, 322, 2720, 22), (STORE, 640, 1632, 22),
+    (STORE, 889, 1168, 42), (RESIDUAL, 889, 1168, 42), (PAIR, 322, 2720, 41), (PAIR, 384, 2720, 41),
+])
+def test_ragged_rounds(epilogue, rows, outs, route):
+    assert qmm_route(epilogue, rows, [outs] * (2 if epilogue == PAIR else 1), 4096) == route
+
+
 def test_k_steps_and_refused_sizes():
     assert qmm_route(STORE, 43, [4096], 320) == 192  # the few-row kernel takes k in steps of 256
     assert qmm_route(STORE, 0, [4096], 4096) == 0
