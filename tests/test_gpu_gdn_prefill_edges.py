@@ -1,7 +1,7 @@
 """Gated DeltaNet prompt kernels against the oracle at the edges of their
 chunks: conv1d around its 16-token chunk and its 3-entry state (the first
 chunk's threads publish the state), the recurrence around its 32-token chunks
-(k.q is formed while a chunk is staged). Bounds as in test_gpu_prefill: state
+(k.q is formed while a chunk is staged, 8 tokens a step). Bounds as in test_gpu_prefill: state
 and outputs of the conv exact / bf16, recurrence outputs bf16, state rel 1e-3."""
 import numpy as np
 import pytest
@@ -29,7 +29,7 @@ def test_conv1d_state_edges(gpu, orc, T, has_prev):
     np.testing.assert_array_equal(sd.numpy(), rs)
 
 
-@pytest.mark.parametrize("T,has_prev", [(31, True), (32, False), (33, True), (95, True)])
+@pytest.mark.parametrize("T,has_prev", [(8, True), (9, False), (24, True), (31, True), (32, False), (33, True), (95, True)])
 def test_recurrence_chunk_edges(gpu, orc, T, has_prev):
     from peregrine_amd import ops
     from peregrine_amd.device import DeviceArray
