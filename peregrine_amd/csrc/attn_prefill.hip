@@ -170,8 +170,10 @@ constexpr float kProbSmall = 0x1p-100f;
 // down to the lane's own four. The first NG groups stay in registers (packed:
 // their f32 values took 256 registers and a wave per SIMD, 260 us) between the
 // two passes; later ones are read again. Bound by reading the scores once
-// (3.2 TB/s). 1600 tokens 16 us, 1021 after 15003 160-179 us, where the softmax
-// that rewrote the row took 49 and 727 us.
+// (3.2 TB/s at a long context); the NG groups are loaded whatever the row's length,
+// so a cold prompt reads the masked half of its rows too (82 MB at 1600 tokens).
+// 1600 tokens 16 us, 1021 after 15003 160-179 us, where the softmax that rewrote
+// the row took 49 and 727 us.
 template <int NG>
 __global__ __launch_bounds__(256) void attn_prefill_stats_kernel(const uint16_t* __restrict__ scores,
                                                                  float2* __restrict__ stats, uint32_t ld, uint32_t T,
@@ -251,10 +253,11 @@ __global__ __launch_bounds__(256) void attn_prefill_stats_kernel(const uint16_t*
 // them to LDS; four consumer waves (2 x 32 rows, 2 x half of the dims) copy the V
 // tiles straight to LDS kBufs - 1 tiles ahead and run the matrix instructions,
 // in slot order from 0, so a row's bits do not depend on the chunk it is
-// computed in. Per tile a producer wave's ~240 VALU operations, the LDS traffic
-// (120 KB) and the matrix instructions (a quarter of the time) meet at one
-// barrier. 1600 tokens 57 -> 46 us, 1021 after 15003 323 -> 245-290 us (a GEMM
-// over stored probabilities before).
+// computed in. A tile takes about 2400 clocks: a producer wave's ~240 VALU
+// operations (960), the LDS traffic (120 KB, as much again) and the matrix
+// instructions (500) follow one another at the tile's barrier rather than overlap.
+// 1600 tokens 57 -> 46.5 us, 1021 after 15003 323 -> 250-290 us (a GEMM over
+// stored probabilities before).
 template <int DS>
 __global__ __launch_bounds__(kPvThreads) void attn_prefill_pv_kernel(const uint16_t* __restrict__ scores,
                                                                      const float2* __restrict__ stats,

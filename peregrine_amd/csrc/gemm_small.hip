@@ -26,8 +26,11 @@ constexpr int kSmallThreads = 512;  // 4 consumer waves, 4 producer waves
 // One barrier per stage. Per output element the instructions are those of
 // gemm_q4_kernel in the same k order (16x16x32 blocks of k 32 i .. +31, one
 // accumulator), so a row has the same bits whichever kernel a call takes.
-// Bound by the producers' dequantisation (about 31 VALU operations per 8
-// values, one wave per SIMD) and the LDS traffic beside it. Measured at 43
+// What bounds it (gate/up at 43 rows, counters): a stage takes about 2200 clocks,
+// of which a producer wave issues VALU operations for 880 (dequantisation, about
+// 31 per 8 values), LDS is busy for 960 (every consumer wave reads all of the
+// dequantised weights) and the matrix cores for 380. Behind one barrier per stage
+// they follow one another instead of overlapping, on 192 of 256 CUs. Measured at 43
 // rows (us, before -> now, 4.5 Q4 bits from HBM): gate/up 12288 x 2 x 4096
 // 57 -> 33; down 4096 x 12288 162 -> 28; 12288 x 4096 55 -> 21; 4096 x 4096
 // 54 -> 13.

@@ -1,6 +1,7 @@
 // Prompt-path (prefill) kernels other than the GEMMs and the attention itself
-// (attn_prefill.hip): attention prepare, conv1d prefill with its state publish, and the Gated DeltaNet prefill (q/k norms + gates, then the
-// token-sequential recurrence).
+// (attn_prefill.hip): attention prepare, conv1d prefill with its state publish,
+// and the Gated DeltaNet prefill (q/k norms + gates, then the token-sequential
+// recurrence).
 //
 // Reference semantics (file:line in the reference tree):
 //   split_qg_many_bf16                       shaders/layout.metal:68-89
@@ -331,8 +332,11 @@ __global__ __launch_bounds__(kPrepWaves * kWave) void gdn_prefill_prepare_kernel
 // staged through LDS in chunks of kGdnChunk tokens, double-buffered: the
 // next chunk's global loads are in flight while the current chunk runs, so the
 // sequential loop only waits on LDS. Outputs collect in LDS and leave once per
-// chunk. (One wave per SIMD: the loop is instruction-issue bound, so a layout
-// with more lanes per row and more waves per SIMD only adds reduction work.)
+// chunk. One wave per SIMD, whose cycles go 54-56% to VALU operations and 26-30%
+// to waits, for the LDS above all: a token takes about 400 clocks, of which LDS
+// is busy for 190 (60 of them bank conflicts), because every row group reads the
+// same q and k. 32 lanes per row and two waves per SIMD took 448 us against 378 at
+// 1600 tokens in an earlier form of this loop.
 constexpr int kGdnPRowsPerBlock = 16;
 constexpr int kGdnChunk = 32;
 
@@ -407,7 +411,8 @@ __global__ __launch_bounds__(256) void gdn_prefill_kernel(float* __restrict__ st
     } else {
       // k.q of the chunk's tokens, four per 32 lanes (each lane its float4 of
       // both): a few operations per chunk instead of 13 per token in the loop
-      // (1600 tokens: 292 -> 267 us).
+      // (1600 tokens: 271 -> 249 us). The model's prompts come with k.q from the
+      // prepare kernel and take the other form (243 us).
       if (tid < kGdnChunk) *reinterpret_cast<float2*>(&sgk[buf][tid]) = make_float2(rg, rbt);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {

@@ -1,8 +1,8 @@
 """Prefill attention against the oracle where its kernels change form: each
 split of the value dims (few, some and many tokens), each register window of
-the row statistics (contexts around 2048, 6144 and past 16384), contexts that
-end inside a 64-slot tile and inside a 16-byte chunk, and cache strides that
-are not a multiple of the tile. Cache slots past the context hold NaN. The
+the row statistics (contexts around 2048, 6144 and past 16384), score blocks of
+2, 3, 4 and 16 tiles, contexts that end inside a 64-slot tile and inside a
+16-byte chunk, and cache strides that are not a multiple of the tile. Cache slots past the context hold NaN. The
 bound is test_gpu_prefill's: one output ulp plus one flipped probability."""
 import numpy as np
 import pytest
@@ -67,7 +67,8 @@ def test_attn_prefill_long_segments_vs_oracle(gpu, orc, T, prefix):
 @pytest.mark.parametrize("T,start,stride", [(1, 0, 8), (63, 5, 72), (64, 0, 64), (65, 100, 168)])
 def test_prepare_aligned_equals_general(gpu, T, start, stride):
     """16-byte aligned operands take the vector kernel, others the general one:
-    the same q, gate and cache bits (slots outside the call's stay untouched)."""
+    the same q, gate and cache bits (slots outside the call's and the memory around
+    each output stay untouched)."""
     from peregrine_amd import ops
     from peregrine_amd.device import DeviceArray
 
@@ -84,7 +85,10 @@ def test_prepare_aligned_equals_general(gpu, T, start, stride):
         p = [a.ptr + 2 * shift for a in arrays]
         ops.attn_prefill_prepare(*p, T, start, start, stride)
         gpu.synchronize()
-        return [a.numpy()[shift:shift + n] for a, n in zip(arrays[5:], sizes)]
+        got = [a.numpy() for a in arrays[5:]]
+        for a, n in zip(got, sizes):  # nothing before or past an output
+            assert not a[:shift].any() and a.size == shift + n + 8 and not a[shift + n:].any()
+        return [a[shift:shift + n] for a, n in zip(got, sizes)]
 
     for a, b, what in zip(run(0), run(1), ("q", "gate", "K cache", "V cache")):
         np.testing.assert_array_equal(a, b, err_msg=what)
