@@ -127,8 +127,8 @@ __global__ __launch_bounds__(kPrepThreads) void attn_prefill_prepare_vec_kernel(
     const uint32_t r = threadIdx.x >> 2, c = (threadIdx.x & 3) * 16;
     if (t0 + r < T) {
       const uint4* src = reinterpret_cast<const uint4*>(v_in + static_cast<size_t>(t0 + r) * kKvDim + d0 + c);
-      const uint4 v[2] = {src[0], src[1]};
-      const uint32_t* p = &v[0].x;
+      const uint4 a = src[0], b = src[1];
+      const uint32_t p[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
       for (uint32_t i = 0; i < 8; ++i) {
         sv[c + 2 * i][r] = static_cast<uint16_t>(p[i]);
