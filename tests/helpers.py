@@ -5,7 +5,7 @@ import numpy as np
 
 from peregrine_amd.synth import bf16_to_f32
 
-# Tolerance stated by the north star for bf16 outputs with fp32 accumulation.
+# Tolerance for bf16 outputs with fp32 accumulation.
 BF16_RTOL = 1e-2
 
 
