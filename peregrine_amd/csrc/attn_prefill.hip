@@ -256,7 +256,7 @@ __global__ __launch_bounds__(256) void attn_prefill_stats_kernel(const uint16_t*
 // computed in. A tile takes about 2400 clocks: a producer wave's ~240 VALU
 // operations (960), the LDS traffic (120 KB, as much again) and the matrix
 // instructions (500) follow one another at the tile's barrier rather than overlap.
-// 1600 tokens 57 -> 46.5 us, 1021 after 15003 323 -> 250-290 us (a GEMM over
+// 1600 tokens 57 -> 46 us, 1021 after 15003 323 -> 250-290 us (a GEMM over
 // stored probabilities before).
 template <int DS>
 __global__ __launch_bounds__(kPvThreads) void attn_prefill_pv_kernel(const uint16_t* __restrict__ scores,
@@ -301,36 +301,71 @@ __global__ __launch_bounds__(kPvThreads) void attn_prefill_pv_kernel(const uint1
 #pragma unroll
       for (int i = 0; i < 2; ++i) ss[set][i] = *reinterpret_cast<const uint4*>(sp[i] + tile * kTileCols);
     };
+    // A tile's probabilities, on straight-line code to the LDS store; where an
+    // exponential or the quotient's residual may underflow (a score 69 or more
+    // under the maximum) the plain division writes them again. A branch before
+    // the store keeps one row's chain from overlapping the other's (9 tokens after
+    // 15000: 165 us). Blocks with a part of the value dims are bound by this chain,
+    // so there the columns past a row's token are zeroed the same way, in the one or
+    // two tiles that have any: 141 us, against 147 with the masks in line and 143
+    // with them and without the test for small exponentials. Blocks with all dims
+    // lose by that (512 after 4000: 111 -> 115 us) and mask in line; the test costs
+    // them 0-1% (1600 tokens 97.1 -> 97.2 us, 1021 after 15003 571 -> 579).
     auto probs = [&](int set, uint32_t tile) {
+      const uint32_t c0 = tile * kTileCols + 8 * pc;
+      auto score = [&](int i, int e) {
+        const uint32_t w = (&ss[set][i].x)[e >> 1];
+        return __fmul_rn((e & 1) ? bf_hi(w) : bf_lo(w), scale);
+      };
+      auto pack = [](const float* p) {
+        return make_uint4(pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7]));
+      };
+      auto put = [&](int i, uint4 v, bool mask) {
+        const uint32_t r = pr + 32 * i;
+        if (mask) {
+          uint32_t* w = &v.x;
+#pragma unroll
+          for (uint32_t e = 0; e < 4; ++e)
+            w[e] &= (c0 + 2 * e <= pvis[i] ? 0xffffu : 0u) | (c0 + 2 * e + 1 <= pvis[i] ? 0xffff0000u : 0u);
+        }
+        sP[tile & 1][r][pc ^ (r & 7)] = v;
+      };
+      uint4 v[2];
+      float least = 1.0f;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const uint32_t w[4] = {ss[set][i].x, ss[set][i].y, ss[set][i].z, ss[set][i].w};
-        const uint32_t c0 = tile * kTileCols + 8 * pc;
-        auto score = [&](int e) { return __fmul_rn((e & 1) ? bf_hi(w[e >> 1]) : bf_lo(w[e >> 1]), scale); };
-        float p[8], least = 1.0f;
+        float p[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const float ex = prob_exp(score(e), pm[i]);
+          const float ex = prob_exp(score(i, e), pm[i]);
           least = fminf(least, ex);
           // ex / sum: the quotient by the rounded reciprocal and one residual step
           // (Markstein). The residual is exact from kProbSmall up; 4e8 random pairs
           // of ex in [2^-100, 1] and sums to 2^17 gave the rounded quotient each time
           const float qt = __fmul_rn(ex, pinv[i]);
           p[e] = __fmaf_rn(__fmaf_rn(-qt, pd[i], ex), pinv[i], qt);
+          if (DS == 1) p[e] = c0 + e <= pvis[i] ? p[e] : 0.0f;
         }
-        // Where the residual or the exponential itself may underflow (a score 69
-        // or more under the maximum): the plain division. Testing the least of
-        // eight costs 1% of the op (1600 tokens 97.1 -> 98.3 us, 1021 after 15003
-        // 570 -> 575); the row's least score from the statistics kernel cost 2%.
-        if (__builtin_expect(least < kProbSmall, 0)) {
+        v[i] = pack(p);
+        put(i, v[i], false);
+      }
+      const bool small = least < kProbSmall;
+      // the tile past the last goes into a buffer nobody reads
+      const bool diag = DS != 1 && tile < tiles && tile * kTileCols + kTileCols - 1 > prefix + t0;
+      if (__builtin_expect(small | diag, 0)) {
+        if (diag) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) p[e] = prob_small(score(e), pm[i], pd[i]);
+          for (int i = 0; i < 2; ++i) put(i, v[i], true);
         }
+        if (small) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) p[e] = c0 + e <= pvis[i] ? p[e] : 0.0f;
-        const uint32_t r = pr + 32 * i;
-        sP[tile & 1][r][pc ^ (r & 7)] =
-            make_uint4(pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7]));
+          for (int i = 0; i < 2; ++i) {
+            float p[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) p[e] = prob_small(score(i, e), pm[i], pd[i]);
+            put(i, pack(p), true);
+          }
+        }
       }
     };
 #pragma unroll
