@@ -253,9 +253,10 @@ __global__ __launch_bounds__(256) void attn_prefill_stats_kernel(const uint16_t*
 // them to LDS; four consumer waves (2 x 32 rows, 2 x half of the dims) copy the V
 // tiles straight to LDS kBufs - 1 tiles ahead and run the matrix instructions,
 // in slot order from 0, so a row's bits do not depend on the chunk it is
-// computed in. A tile takes about 2400 clocks: a producer wave's ~240 VALU
-// operations (960), the LDS traffic (120 KB, as much again) and the matrix
-// instructions (500) follow one another at the tile's barrier rather than overlap.
+// computed in. A tile takes about 2000 clocks (counters, long context): a producer
+// wave's ~240 VALU operations take 960, the matrix cores are busy for 510 and LDS
+// reads and stores for 380 beside the V copies; behind one barrier per tile they
+// mostly follow one another.
 // 1600 tokens 57 -> 46 us, 1021 after 15003 323 -> 250-290 us (a GEMM over
 // stored probabilities before).
 template <int DS>

@@ -333,7 +333,7 @@ __global__ __launch_bounds__(kPrepWaves * kWave) void gdn_prefill_prepare_kernel
 // next chunk's global loads are in flight while the current chunk runs, so the
 // sequential loop only waits on LDS. Outputs collect in LDS and leave once per
 // chunk. One wave per SIMD, whose cycles go 54-56% to VALU operations and 26-30%
-// to waits, for the LDS above all: a token takes about 400 clocks, of which LDS
+// to waits, for the LDS above all: a token takes about 365 clocks, of which LDS
 // is busy for 190 (60 of them bank conflicts), because every row group reads the
 // same q and k. 32 lanes per row and two waves per SIMD took 448 us against 378 at
 // 1600 tokens in an earlier form of this loop.
